@@ -76,3 +76,55 @@ def test_small_workspace_keeps_the_plan_over_requests():
     out = small.run(b.q, b.cache)
     ref = AP.oracle_per_request(b, "causal")[None]
     AP.check(out, ref[0])
+
+
+def _exact64(b, r):
+    """float64 output [qo_len, heads, D] of request r (causal)."""
+    q0, q1 = int(b.qo_indptr[r]), int(b.qo_indptr[r + 1])
+    pages = b.kv_indices[int(b.kv_indptr[r]):int(b.kv_indptr[r + 1])].long()
+    L, n, g = int(b.kv_lens[r]), q1 - q0, b.num_qo_heads // b.num_kv_heads
+    kv = b.cache[pages]
+    seen = torch.arange(L, device=DEV) <= torch.arange(n, device=DEV)[:, None, None] + L - n
+    out = torch.empty((n, b.num_qo_heads, b.head_dim), dtype=torch.float64, device=DEV)
+    for h in range(b.num_kv_heads):
+        k = kv[:, 0, :, h].reshape(-1, b.head_dim)[:L].double()
+        v = kv[:, 1, :, h].reshape(-1, b.head_dim)[:L].double()
+        q = b.q[q0:q1, h * g:(h + 1) * g].double().reshape(n * g, b.head_dim)
+        s = (q @ k.t().contiguous() / b.head_dim ** 0.5).reshape(n, g, L)
+        p = torch.softmax(s.masked_fill(~seen, -torch.inf), -1).reshape(n * g, L)
+        out[:, h * g:(h + 1) * g] = (p @ v).reshape(n, g, b.head_dim)
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_blocks_lose_no_precision(dtype):
+    """Query tokens whose block is split although the plan over requests runs their request
+    whole: the error against 64 bits is that of the unsplit output.  The parts add fp32
+    roundings (2^-24) to an output rounded to 2^-9 or 2^-12; the bound leaves 2% for the
+    softmax weights' rounding, which falls differently (a second rounding to the 16-bit
+    type makes it about 1.2 times)."""
+    b = make_verify_batch(4, 0, 0, 0, 32, 8, 128, 16, dtype=dtype, scale=0.5, seed=41,
+                          qo_lens=np.full(4, 512), ctx=np.full(4, 1024), device=DEV)
+    args = (b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, 32, 8, 128, 16)
+
+    def planned(nbytes):
+        w = bsx.BatchPrefillWithPagedKVCacheWrapper(
+            torch.empty(nbytes, dtype=torch.uint8, device=DEV), "NHD")
+        w.plan(*args, causal=True, q_data_type=dtype)
+        return w
+
+    blocks = planned(256 << 20)
+    p = blocks.plan_info
+    assert p.block_batch > 0 and p.num_split_requests > 0
+    whole = planned(blocks._blob_bytes)  # no room for partials
+    assert whole.plan_info.block_batch == 0 and whole.plan_info.num_split_requests == 0
+    rec = blocks.plan_blob[p.off_merge_seqs:p.off_merge_seqs + 4 * p.num_split_requests]
+    split = torch.zeros(b.q.shape[0], dtype=torch.bool, device=DEV)
+    for _, _, q0, n in rec.reshape(-1, 4):
+        split[int(q0):int(q0) + int(n)] = True
+    ref = torch.cat([_exact64(b, r) for r in range(4)])[split]
+    err = [float((w.run(b.q, b.cache).double()[split] - ref).norm() / ref.norm())
+           for w in (whole, blocks)]
+    print(f"split query tokens {int(split.sum())} of {len(split)}: relative error whole "
+          f"{err[0]:.6f}, blocks {err[1]:.6f}", flush=True)
+    assert err[1] <= 1.02 * err[0]

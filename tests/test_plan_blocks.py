@@ -63,7 +63,7 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
             for s in mine:
                 rows_used += list(range(s[3], s[3] + ql * g))
     assert sorted(rows_used) == list(range(plan.part_rows))
-    assert plan.float_ws_bytes == plan.part_rows * hkv * (128 * 2 + 4)
+    assert plan.float_ws_bytes == plan.part_rows * hkv * (128 * 4 + 4)  # fp32 partials
 
 
 def test_rule_and_workspace_fallback():
