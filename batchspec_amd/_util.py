@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import functools
+import threading
 
 import torch
 
@@ -54,23 +55,42 @@ def num_cus(device_index: int) -> int:
     return torch.cuda.get_device_properties(device_index).multi_processor_count
 
 
-def workspace(device: torch.device, nbytes: int, cache: dict | None = None,
-              key: str = "ws") -> torch.Tensor:
-    """A uint8 device buffer of at least `nbytes`, reused through `cache`.
+# Held from a call's choice of a workspace until its launches are queued: the launches of
+# one call share the workspace, so two host threads on one stream must not interleave theirs
+# (ctypes releases the GIL during the call).
+LAUNCH_LOCK = threading.Lock()
 
-    A buffer that is outgrown is never freed: a graph captured while it was current
-    holds its address as a kernel argument, and replaying that graph must not write
-    into memory the caching allocator has handed to another tensor.  Growth doubles,
-    so the retired buffers together stay below the current one."""
+
+_MAX_WORKSPACES = 64  # eager ones of a cache: torch has 32 pooled streams
+
+
+def workspace(device: torch.device, nbytes: int, cache: dict, name: str,
+              stream: int) -> torch.Tensor:
+    """A uint8 device buffer of at least `nbytes`, reused through `cache` by the calls of
+    `name` on this device and stream, which must be the current one (the caller holds
+    LAUNCH_LOCK).
+
+    One per stream: a call's kernels hand results to each other through it, and calls on
+    different streams may run at the same time.  Dropping one is safe: the allocator gives
+    its memory only to later work on the same stream.
+    Captured calls take buffers of their own, since a graph may replay beside eager work on
+    any stream, and those are never freed ("__retired__"): the graph holds their addresses
+    as kernel arguments.  Growth doubles, so the outgrown ones stay below the current one.
+    Graphs captured on one stream share a buffer: their replays must not overlap."""
     nbytes = max(int(nbytes), 256)
-    if cache is None:
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    captured = torch.cuda.is_current_stream_capturing()
+    key = (name, device.index, stream, captured)
     buf = cache.get(key)
-    if buf is not None and buf.numel() >= nbytes and buf.device == device:
+    if buf is not None and buf.numel() >= nbytes:
         return buf
     if buf is not None:
-        cache.setdefault("__retired__", []).append(buf)
         nbytes = max(nbytes, 2 * buf.numel())
     buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if captured:
+        cache.setdefault("__retired__", []).append(buf)
+    else:
+        eager = [k for k in cache if k != "__retired__" and not k[3] and k != key]
+        if len(eager) >= _MAX_WORKSPACES:
+            del cache[eager[0]]
     cache[key] = buf
     return buf

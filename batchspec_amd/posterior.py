@@ -21,7 +21,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._util import dtype_code, require_gpu, stream_of, workspace
+from ._util import LAUNCH_LOCK, dtype_code, require_gpu, stream_of, workspace
 from .sampling import _uniforms
 
 _WS: dict = {}
@@ -63,12 +63,14 @@ def _sampled(draft: torch.Tensor, logits: torch.Tensor, eos: int, temperature: f
     accept = torch.empty(B, dtype=torch.int32, device=dev)
     eos_acc = torch.empty((B, 1), dtype=torch.bool, device=dev)
     lib = _lib.load()
-    ws = workspace(dev, int(lib.bsx_accept_sampling_ws_bytes(B, k, V)), _WS, f"sampling:{dev}")
     x = logits.contiguous()
-    rc = lib.bsx_accept_sampling(ids.data_ptr(), x.data_ptr(), dtype_code(x.dtype),
-                                 float(temperature), int(top_k), float(top_p), u.data_ptr(), B, k,
-                                 V, int(eos), bonus.data_ptr(), accept.data_ptr(),
-                                 eos_acc.data_ptr(), ws.data_ptr(), ws.numel(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = workspace(dev, int(lib.bsx_accept_sampling_ws_bytes(B, k, V)), _WS, "sampling", st)
+        rc = lib.bsx_accept_sampling(ids.data_ptr(), x.data_ptr(), dtype_code(x.dtype),
+                                     float(temperature), int(top_k), float(top_p), u.data_ptr(), B,
+                                     k, V, int(eos), bonus.data_ptr(), accept.data_ptr(),
+                                     eos_acc.data_ptr(), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "evaluate_posterior")
     return bonus, accept, eos_acc
 
@@ -93,10 +95,12 @@ def _greedy(draft: torch.Tensor, preds: torch.Tensor, eos: int, mode: int):
             raise ValueError(f"target logits must be [B, k+1, V], got {tuple(preds.shape)}")
         V = preds.shape[2]
         x = preds.contiguous()
-        ws = workspace(dev, int(lib.bsx_accept_greedy_ws_bytes(B, k, V)), _WS, f"greedy:{dev}")
-        rc = lib.bsx_accept_greedy(d.data_ptr(), None, x.data_ptr(), dtype_code(x.dtype), B, k, V,
-                                   int(eos), mode, bonus.data_ptr(), accept.data_ptr(),
-                                   eos_acc.data_ptr(), ws.data_ptr(), ws.numel(), stream_of(dev))
+        st = stream_of(dev)
+        with LAUNCH_LOCK:
+            ws = workspace(dev, int(lib.bsx_accept_greedy_ws_bytes(B, k, V)), _WS, "greedy", st)
+            rc = lib.bsx_accept_greedy(d.data_ptr(), None, x.data_ptr(), dtype_code(x.dtype), B, k,
+                                       V, int(eos), mode, bonus.data_ptr(), accept.data_ptr(),
+                                       eos_acc.data_ptr(), ws.data_ptr(), ws.numel(), st)
     else:
         raise ValueError("target_preds must be ids [B, k+1] or logits [B, k+1, V]")
     _lib.check(rc, "evaluate_posterior")
@@ -123,7 +127,7 @@ def evaluate_posterior_and_delete(draft_tokens: torch.Tensor, target_preds: torc
     eos_acc = torch.empty(B, dtype=torch.uint8, device=dev)
     lib = _lib.load()
     ids = logits = None
-    V, dt, ws = 0, 0, None
+    V, dt, need = 0, 0, 0
     if target_preds.dim() == 2:
         if target_preds.shape != (B, k + 1):
             raise ValueError(f"target ids must be [B, k+1], got {tuple(target_preds.shape)}")
@@ -133,17 +137,20 @@ def evaluate_posterior_and_delete(draft_tokens: torch.Tensor, target_preds: torc
             raise ValueError(f"target logits must be [B, k+1, V], got {tuple(target_preds.shape)}")
         logits = target_preds.contiguous()
         V, dt = logits.shape[2], dtype_code(logits.dtype)
-        ws = workspace(dev, int(lib.bsx_accept_greedy_ws_bytes(B, k, V)), _WS, f"greedy:{dev}")
+        need = int(lib.bsx_accept_greedy_ws_bytes(B, k, V))
     else:
         raise ValueError("target_preds must be ids [B, k+1] or logits [B, k+1, V]")
     pt = page_table
-    rc = lib.bsx_accept_greedy_delete(
-        d.data_ptr(), _lib.ptr(ids), _lib.ptr(logits), dt, B, k, V, int(eos_token_id),
-        _RULES[accept_rule], bonus.data_ptr(), accept.data_ptr(), eos_acc.data_ptr(),
-        _lib.ptr(ws), 0 if ws is None else ws.numel(), int(n_inserted),
-        pt.page_manager.num_allocated_pages.data_ptr(), pt.paged_kv_last_page_len.data_ptr(),
-        pt.cachelens.data_ptr(), pt.page_size, pt.max_num_pages_per_request,
-        pt.paged_kv_indptr.data_ptr(), pt.paged_kv_indices.data_ptr(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = None if logits is None else workspace(dev, need, _WS, "greedy", st)
+        rc = lib.bsx_accept_greedy_delete(
+            d.data_ptr(), _lib.ptr(ids), _lib.ptr(logits), dt, B, k, V, int(eos_token_id),
+            _RULES[accept_rule], bonus.data_ptr(), accept.data_ptr(), eos_acc.data_ptr(),
+            _lib.ptr(ws), 0 if ws is None else ws.numel(), int(n_inserted),
+            pt.page_manager.num_allocated_pages.data_ptr(), pt.paged_kv_last_page_len.data_ptr(),
+            pt.cachelens.data_ptr(), pt.page_size, pt.max_num_pages_per_request,
+            pt.paged_kv_indptr.data_ptr(), pt.paged_kv_indices.data_ptr(), st)
     _lib.check(rc, "evaluate_posterior_and_delete")
     return bonus[:, None], accept, eos_acc.view(torch.bool)[:, None]
 

@@ -26,13 +26,13 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._util import dtype_code, require_gpu, stream_of, workspace
+from ._util import LAUNCH_LOCK, dtype_code, require_gpu, stream_of, workspace
 
 _WS: dict = {}
 
 
-def _ws(dev: torch.device, nbytes: int, key: str) -> torch.Tensor:
-    return workspace(dev, nbytes, _WS, f"{key}:{dev}")
+def _ws(dev: torch.device, nbytes: int, name: str, stream: int) -> torch.Tensor:
+    return workspace(dev, nbytes, _WS, name, stream)
 
 
 def _uniforms(B: int, k: int, dev, uniforms: Optional[torch.Tensor],
@@ -83,13 +83,14 @@ def chain_speculative_sampling(draft_probs: Optional[torch.Tensor], draft_token_
     emi = torch.empty(B, dtype=torch.int32, device=dev)
     lib = _lib.load()
     need = int(lib.bsx_chain_ws_bytes(B, k, V))
-    ws = _ws(dev, need, "chain")
     tp = target_probs.contiguous()
     dp = None if draft_probs is None else draft_probs.contiguous()
-    rc = lib.bsx_chain_speculative_sampling(_lib.ptr(dp), ids.data_ptr(), tp.data_ptr(),
-                                            u.data_ptr(), B, k, V, out.data_ptr(), acc.data_ptr(),
-                                            emi.data_ptr(), ws.data_ptr(), ws.numel(),
-                                            stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, need, "chain", st)
+        rc = lib.bsx_chain_speculative_sampling(
+            _lib.ptr(dp), ids.data_ptr(), tp.data_ptr(), u.data_ptr(), B, k, V, out.data_ptr(),
+            acc.data_ptr(), emi.data_ptr(), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "chain_speculative_sampling")
     return (out, _accumulate(maybe_output_accepted_token_num, acc),
             _accumulate(maybe_output_emitted_draft_token_num, emi))
@@ -124,13 +125,16 @@ def chain_speculative_sampling_from_logits(draft_logits: Optional[torch.Tensor],
     acc = torch.empty(B, dtype=torch.int32, device=dev)
     emi = torch.empty(B, dtype=torch.int32, device=dev)
     lib = _lib.load()
-    ws = _ws(dev, int(lib.bsx_chain_filtered_ws_bytes(B, k, V)), "chain")
+    need = int(lib.bsx_chain_filtered_ws_bytes(B, k, V))
     tl = target_logits.contiguous()
     dl = None if draft_logits is None else draft_logits.contiguous()
-    rc = lib.bsx_chain_speculative_sampling_filtered(
-        _lib.ptr(dl), ids.data_ptr(), tl.data_ptr(), dtype_code(tl.dtype), float(temperature),
-        int(top_k), float(top_p), u.data_ptr(), B, k, V, out.data_ptr(), acc.data_ptr(),
-        emi.data_ptr(), ws.data_ptr(), ws.numel(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, need, "chain", st)
+        rc = lib.bsx_chain_speculative_sampling_filtered(
+            _lib.ptr(dl), ids.data_ptr(), tl.data_ptr(), dtype_code(tl.dtype), float(temperature),
+            int(top_k), float(top_p), u.data_ptr(), B, k, V, out.data_ptr(), acc.data_ptr(),
+            emi.data_ptr(), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "chain_speculative_sampling_from_logits")
     return out, acc, emi
 
@@ -147,9 +151,11 @@ def softmax(logits: torch.Tensor, temperature: Optional[float] = None,
         raise ValueError("temperature must be > 0")
     probs = torch.empty(logits.shape, dtype=torch.float32, device=dev)
     lib = _lib.load()
-    ws = _ws(dev, int(lib.bsx_softmax_ws_bytes(rows)), "softmax")
-    rc = lib.bsx_softmax(x.data_ptr(), dtype_code(x.dtype), T, rows, V, probs.data_ptr(),
-                         ws.data_ptr(), ws.numel(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, int(lib.bsx_softmax_ws_bytes(rows)), "softmax", st)
+        rc = lib.bsx_softmax(x.data_ptr(), dtype_code(x.dtype), T, rows, V, probs.data_ptr(),
+                             ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "softmax")
     return probs
 
@@ -162,9 +168,11 @@ def argmax(logits: torch.Tensor) -> torch.Tensor:
     rows = x.numel() // V
     out = torch.empty(logits.shape[:-1], dtype=torch.int64, device=dev)
     lib = _lib.load()
-    ws = _ws(dev, int(lib.bsx_argmax_ws_bytes(rows, V)), "argmax")
-    rc = lib.bsx_argmax(x.data_ptr(), dtype_code(x.dtype), rows, V, V, out.data_ptr(),
-                        ws.data_ptr(), ws.numel(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, int(lib.bsx_argmax_ws_bytes(rows, V)), "argmax", st)
+        rc = lib.bsx_argmax(x.data_ptr(), dtype_code(x.dtype), rows, V, V, out.data_ptr(),
+                            ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "argmax")
     return out
 
@@ -190,10 +198,12 @@ def get_sampling_probs(logits: torch.Tensor, top_p: float, top_k: int,
     rows, V = x.shape
     probs = torch.empty((rows, V), dtype=torch.float32, device=dev)
     lib = _lib.load()
-    ws = _ws(dev, int(lib.bsx_sampling_probs_ws_bytes(rows)), "probs")
-    rc = lib.bsx_sampling_probs(x.data_ptr(), dtype_code(x.dtype), float(temperature), int(top_k),
-                                float(top_p), rows, V, probs.data_ptr(), ws.data_ptr(), ws.numel(),
-                                stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, int(lib.bsx_sampling_probs_ws_bytes(rows)), "probs", st)
+        rc = lib.bsx_sampling_probs(x.data_ptr(), dtype_code(x.dtype), float(temperature),
+                                    int(top_k), float(top_p), rows, V, probs.data_ptr(),
+                                    ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "get_sampling_probs")
     return probs.reshape(B, S, V)
 
@@ -220,9 +230,11 @@ def sample(logits: torch.Tensor, top_p: float, top_k: int, temperature: float, *
         u = uniforms.reshape(rows).contiguous()
     ids = torch.empty((B, S), dtype=torch.int64, device=dev)
     lib = _lib.load()
-    ws = _ws(dev, int(lib.bsx_sample_ids64_ws_bytes(rows, V)), "sample")
-    rc = lib.bsx_sample_ids64(x.data_ptr(), dtype_code(x.dtype), float(temperature), int(top_k),
-                              float(top_p), u.data_ptr(), rows, V, ids.data_ptr(), ws.data_ptr(),
-                              ws.numel(), stream_of(dev))
+    st = stream_of(dev)
+    with LAUNCH_LOCK:
+        ws = _ws(dev, int(lib.bsx_sample_ids64_ws_bytes(rows, V)), "sample", st)
+        rc = lib.bsx_sample_ids64(x.data_ptr(), dtype_code(x.dtype), float(temperature),
+                                  int(top_k), float(top_p), u.data_ptr(), rows, V, ids.data_ptr(),
+                                  ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "sample")
     return ids
