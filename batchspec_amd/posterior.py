@@ -16,13 +16,14 @@ Same inputs and outputs as MTPEngine.evaluate_posterior
 """
 from __future__ import annotations
 
+import numbers
 from typing import Optional, Tuple
 
 import torch
 
 from . import _lib
 from ._util import LAUNCH_LOCK, dtype_code, require_gpu, stream_of, workspace
-from .sampling import _uniforms
+from .sampling import _uniforms, chain_speculative_sampling_from_logits
 
 _WS: dict = {}
 _RULES = {"reference": 0, "prefix": 1}
@@ -39,8 +40,17 @@ def evaluate_posterior(draft_tokens: torch.Tensor, target_preds: torch.Tensor, *
         return _greedy(draft_tokens, target_preds, eos_token_id, _RULES[accept_rule])
     if target_preds.dim() != 3:
         raise ValueError("sampling acceptance needs target logits [B, k+1, V]")
-    return _sampled(draft_tokens, target_preds, eos_token_id, temperature, top_p, top_k, uniforms,
-                    generator)
+    if isinstance(eos_token_id, numbers.Integral):
+        return _sampled(draft_tokens, target_preds, int(eos_token_id), temperature, top_p, top_k,
+                        uniforms, generator)
+    # an eos id that the kernel does not take (a tensor, also one id per request; a float)
+    # compares as torch compares it
+    out, _, emitted = chain_speculative_sampling_from_logits(
+        None, draft_tokens, target_preds, temperature, generator, uniforms=uniforms,
+        top_k=top_k, top_p=top_p)
+    last = (out != -1).to(torch.long) * torch.arange(out.shape[1], device=out.device)
+    bonus = out.gather(1, last.argmax(dim=1, keepdim=True))
+    return bonus, emitted + 1, (out == eos_token_id).any(dim=1, keepdim=True)
 
 
 def _sampled(draft: torch.Tensor, logits: torch.Tensor, eos: int, temperature: float,
@@ -54,7 +64,7 @@ def _sampled(draft: torch.Tensor, logits: torch.Tensor, eos: int, temperature: f
         raise ValueError(f"target_logits must be [B, k+1, V], got {tuple(logits.shape)}")
     if not temperature > 0:
         raise ValueError("temperature must be > 0 (greedy acceptance: evaluate_posterior)")
-    if not -2 ** 31 <= int(eos) < 2 ** 31:
+    if not -2 ** 31 <= eos < 2 ** 31:
         raise RuntimeError(f"eos_token_id {eos} is outside the int32 token ids")
     V = logits.shape[2]
     ids = draft.to(torch.int64).contiguous()
@@ -69,7 +79,7 @@ def _sampled(draft: torch.Tensor, logits: torch.Tensor, eos: int, temperature: f
         ws = workspace(dev, int(lib.bsx_accept_sampling_ws_bytes(B, k, V)), _WS, "sampling", st)
         rc = lib.bsx_accept_sampling(ids.data_ptr(), x.data_ptr(), dtype_code(x.dtype),
                                      float(temperature), int(top_k), float(top_p), u.data_ptr(), B,
-                                     k, V, int(eos), bonus.data_ptr(), accept.data_ptr(),
+                                     k, V, eos, bonus.data_ptr(), accept.data_ptr(),
                                      eos_acc.data_ptr(), ws.data_ptr(), ws.numel(), st)
     _lib.check(rc, "evaluate_posterior")
     return bonus, accept, eos_acc

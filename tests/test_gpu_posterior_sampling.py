@@ -45,3 +45,21 @@ def test_sampling_verdict(case):
         assert got[0].dtype == torch.int32 and got[1].dtype == torch.int32
         assert torch.equal(got[0], bonus) and torch.equal(got[1], emitted + 1)
         assert torch.equal(got[2], (out == eos).any(dim=1, keepdim=True))
+
+
+def test_sampling_verdict_other_eos_ids():
+    """An eos id that is not a plain integer compares as torch compares it: a tensor of one
+    id, a tensor of one id per request, and floats, equal to an id or not."""
+    B, k, V = 6, 3, 3000
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    logits = torch.randn((B, k + 1, V), generator=gen, device=DEV) * 4
+    draft = logits[:, :k].argmax(-1)
+    u = torch.rand((B, k + 1), generator=gen, device=DEV)
+    out, _, emitted = chain_speculative_sampling_from_logits(None, draft, logits, 0.8, uniforms=u)
+    hit = int(out[0, 0])
+    for eos in (torch.tensor(hit, device=DEV), out[:, :1].clone(), float(hit), hit + 0.5, 1e30):
+        got = evaluate_posterior(draft, logits, greedy=False, eos_token_id=eos, temperature=0.8,
+                                 uniforms=u)
+        assert torch.equal(got[2], (out == eos).any(dim=1, keepdim=True))
+        assert torch.equal(got[1], emitted + 1)
+        assert got[0].dtype == torch.int32 and got[1].dtype == torch.int32
