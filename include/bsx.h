@@ -77,7 +77,7 @@ typedef struct {
   int32_t mask_mode;
   int32_t group_size;     /* num_qo_heads / num_kv_heads                      */
   int32_t qrow_tile;      /* query rows per wave (16 or 32)                   */
-  int32_t qrow_blocks;    /* waves per kv head that split the query rows      */
+  int32_t qrow_blocks;    /* waves per kv head that split a record's query rows */
   int32_t heads_per_cta;  /* kv heads handled by one workgroup                */
   int32_t qblocks_per_cta;/* query-row blocks handled by one workgroup        */
   int32_t num_qgroups;    /* ceil(qrow_blocks / qblocks_per_cta)              */
@@ -112,12 +112,10 @@ typedef struct {
                              bsx_attn_plan_device; counts above are bounds    */
   int32_t off_dyn;        /* device plan: int32 offset of {split requests,
                              error code, segments, reserved} in the blob      */
-  int32_t block_batch;    /* > 0: the schedule's records are blocks of at most
-                             128 query rows of a request (several per long
-                             request, each with the kv tokens its rows can
-                             see), run by workgroups of 4 waves; grid.y =
-                             num_kv_heads, and qblocks_per_cta and num_qgroups
-                             only describe the plan over whole requests.
+  int32_t block_batch;    /* > 0: the schedule's records are this many blocks
+                             of at most 128 query rows of a request (several per
+                             long request, each with the kv tokens its rows can
+                             see): qblocks_per_cta 4, num_qgroups 1.
                              0: one record per request                         */
   int32_t part_rows;      /* block plans: rows per kv head of all partials (the
                              partials are packed: slots count rows)            */

@@ -90,10 +90,11 @@ def test_query_lengths(qo):
 # through LDS: (D, Hq, Hkv, qo, page size, dtype, ctx range, causal, waves per head).
 SHARED_CASES = [
     (64, 32, 4, 12, 32, torch.float16, (100, 2000), True, 4),
-    (64, 16, 2, 40, 16, torch.bfloat16, (50, 1500), True, 8),   # two query groups
+    (64, 16, 2, 40, 16, torch.bfloat16, (50, 1500), True, 4),   # query blocks
     (128, 32, 8, 24, 64, torch.float16, (8000, 20000), True, 4),  # split + merge
     (128, 32, 8, 33, 16, torch.bfloat16, (40, 3000), False, 8),
     (128, 32, 8, 16, 16, torch.bfloat16, (1, 700), True, 2),
+    (64, 16, 2, 40, 16, torch.bfloat16, (50, 1500), False, 8),  # two query groups
 ]
 
 
@@ -105,6 +106,8 @@ def test_shared_kv_tiles(case):
                           seed=300 + case).to(DEV)
     out, w = run_gpu(b, causal=causal)
     assert w.plan_info.shared_kv_tiles == 1 and w.plan_info.qblocks_per_cta == qb
+    assert (w.plan_info.block_batch > 0) == (causal and qo * Hq // Hkv > 256)
+    assert w.plan_info.num_qgroups == (2 if qb == 8 and qo * Hq // Hkv > 256 else 1)
     check(out, oracle_out(b, "causal" if causal else "none"))
 
 
@@ -129,7 +132,7 @@ def test_continuous_batching_mix(dtype):
     b = make_verify_batch(8, 0, 0, 0, 32, 8, 128, 16, dtype=dtype, scale=0.5, seed=19,
                           qo_lens=qo, ctx=ctx).to(DEV)
     out, w = run_gpu(b)
-    assert w.plan_info.shared_kv_tiles == 1 and w.plan_info.num_qgroups == 2
+    assert w.plan_info.shared_kv_tiles == 1 and w.plan_info.block_batch > 0
     check(out, oracle_out(b, "causal"))
 
 

@@ -67,11 +67,7 @@ def test_small_workspace_keeps_the_plan_over_requests():
     need = big._blob_bytes + int(big.plan_info.float_ws_bytes)
     small = bsx.BatchPrefillWithPagedKVCacheWrapper(
         torch.empty(need - 1, dtype=torch.uint8, device=DEV), "NHD")
-    try:
-        small.plan(*args, causal=True, q_data_type=b.q.dtype)
-    except ValueError as e:  # the plan over requests does not fit either
-        assert "float_workspace_buffer too small" in str(e)
-        return
+    small.plan(*args, causal=True, q_data_type=b.q.dtype)
     assert small.plan_info.block_batch == 0
     out = small.run(b.q, b.cache)
     ref = AP.oracle_per_request(b, "causal")[None]

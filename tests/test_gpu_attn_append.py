@@ -107,15 +107,60 @@ def test_tree_small_pages_and_query_groups():
     ws = _wrapper(s, causal=True)
     got, want = _both(s, ws)
     _equal(got, want, "page size 8")
-    for ps in (16, 8):  # 80 drafts x group 4 = 320 rows: two query groups per kv head
+    for ps in (16, 8):  # 80 drafts x group 4 = 320 rows: query blocks, two query groups
         d = make_verify_batch(4, 200, 3000, 80, 32, 8, 128, ps, dtype=torch.bfloat16,
                               seed=11 + ps, device=DEV)
         wd = _wrapper(d, causal=True)
-        assert wd.plan_info.num_qgroups > 1
+        assert wd.plan_info.num_qgroups > 1 if ps == 8 else wd.plan_info.block_batch > 0
         got, want = _both(d, wd)
-        _equal(got, want, f"two query groups, page size {ps}")
+        _equal(got, want, f"320 query rows, page size {ps}")
         ref = AP.oracle_per_request(_with_cache(d, want[2]), "causal")[None]
         AP.check(got[0], ref[0], got[1], ref[1])
+
+
+@pytest.mark.parametrize("how", ["graph", "device", "workspace"])
+@pytest.mark.parametrize("hq,hkv,d,qo,ctx", [
+    (16, 2, 64, [40, 33, 1, 5], [50, 1500, 700, 3000]),          # 320 rows, a group that idles
+    (32, 8, 128, [128, 80, 5], [965, 2158, 1782]),               # 512 rows
+])
+def test_causal_query_groups_of_whole_requests(how, hq, hkv, d, qo, ctx):
+    """Causal plans with several query groups that keep a record per request: those of graph
+    mode, device plans, and host plans whose workspace does not hold a block plan's partials.
+    The fused update against the two calls, and both against the oracle."""
+    say(f"causal query groups of whole requests ({how}): H={hq}/{hkv} D={d} qo={qo} ctx={ctx}")
+    b = make_verify_batch(len(qo), 0, 0, 0, hq, hkv, d, 16, dtype=torch.bfloat16, scale=0.5,
+                          seed=60 + hq, qo_lens=np.array(qo), ctx=np.array(ctx), device=DEV)
+    q, k, v = b.q, b.k_new, b.v_new
+    if how == "graph":
+        w = bsx.BatchPrefillWithPagedKVCacheWrapper(
+            torch.empty(256 << 20, dtype=torch.uint8, device=DEV), "NHD", use_cuda_graph=True,
+            qo_indptr_buf=b.qo_indptr.clone(), paged_kv_indptr_buf=b.kv_indptr.clone(),
+            paged_kv_indices_buf=b.kv_indices.clone(),
+            paged_kv_last_page_len_buf=b.kv_last_page_len.clone())
+        w.plan(b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, hq, hkv, d, 16,
+               causal=True, q_data_type=b.q.dtype)
+    elif how == "device":
+        w = _wrapper(b, causal=True, on_device=True, max_qo=max(qo))
+        rows = len(qo) * max(qo)  # a device plan takes its bound of query rows
+        pad = lambda x: torch.cat([x, x.new_zeros((rows - x.shape[0], *x.shape[1:]))])
+        q, k, v = pad(q), pad(k), pad(v)
+    else:
+        blocks = _wrapper(b, causal=True)
+        assert blocks.plan_info.block_batch > 0 and blocks.plan_info.float_ws_bytes > 0
+        w = bsx.BatchPrefillWithPagedKVCacheWrapper(
+            torch.empty(blocks._blob_bytes + int(blocks.plan_info.float_ws_bytes) - 1,
+                        dtype=torch.uint8, device=DEV), "NHD")
+        w.plan(b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, hq, hkv, d, 16,
+               causal=True, q_data_type=b.q.dtype)
+    p = w.plan_info
+    assert p.block_batch == 0 and p.shared_kv_tiles == 1
+    assert p.qblocks_per_cta == 8 and p.num_qgroups == 2
+    got, want = _both(b, w, q, k, v)
+    n = b.q.shape[0]
+    got, want = [[t[0][:n], t[1][:n], t[2]] for t in (got, want)]
+    _equal(got, want, how)
+    ref = AP.oracle_per_request(_with_cache(b, want[2]), "causal")[None]
+    AP.check(got[0], ref[0], got[1], ref[1])
 
 
 def test_streaming_view_with_append():

@@ -38,12 +38,16 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
     plan, blob, qoi, kvp = _plan(qo, kv, hq, hkv)
     g = hq // hkv
     n = plan.block_batch
-    assert n > 0 and plan.num_qgroups > 1
+    assert n > 0
+    # the launched workgroups: 4 waves of 32 query rows on one kv head, one per (share, head)
+    assert (plan.qrow_tile, plan.qblocks_per_cta, plan.qrow_blocks) == (32, 4, 4)
+    assert plan.num_qgroups == 1 and plan.heads_per_cta == 1
+    assert plan.num_ctas * hkv <= 2 * 256
     seq = blob[:4 * n].reshape(-1, 4)
     segs = blob[plan.off_segments:plan.off_segments + 4 * plan.num_segments].reshape(-1, 4)
     token_owner = np.zeros(int(qoi[-1]), int)
     for q0, ql, kl, ps0 in seq:
-        assert 0 < ql * g <= plan.qrow_tile * plan.qblocks_per_cta
+        assert 0 < ql * g <= 4 * 32
         token_owner[q0:q0 + ql] += 1
         r = int(np.searchsorted(qoi, q0, side="right")) - 1
         while qo[r] == 0:
@@ -73,7 +77,8 @@ def test_rule_and_workspace_fallback():
     for mode in (_lib.MASK_NONE, _lib.MASK_CUSTOM):
         assert _plan(qo, kv, 32, 8, mode=mode)[0].block_batch == 0
     assert _plan(qo, kv, 32, 8, ps=8)[0].block_batch == 0      # pages below 16 tokens
-    assert _plan([64, 5], kv, 32, 8)[0].block_batch == 0       # one block holds the longest
+    # 64 * 4 query rows: one 8-wave workgroup of the plan over requests holds the longest
+    assert _plan([64, 5], kv, 32, 8)[0].block_batch == 0
     whole = _plan(qo, kv, 32, 8, ws=0)[0]
     assert blk.float_ws_bytes == 0 or whole.block_batch == 0
     strict = _plan(qo, kv, 32, 8, ws=None)[0]
