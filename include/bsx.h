@@ -143,7 +143,10 @@ int bsx_attn_plan(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
                   bsx_attn_plan_t* plan_out);
 
 /* bsx_attn_plan for a caller whose float workspace holds float_ws_capacity bytes: a
- * plan over query blocks (block_batch > 0) is taken when its partials fit there.
+ * plan over query blocks (block_batch > 0) is taken when its partials fit there and its
+ * records fit a blob of bsx_attn_plan_ints_bound entries (about 4000 blocks at 256 compute
+ * units and a small batch, so 1 request of 64000 query tokens at 64/8 heads; more query
+ * tokens keep one record per request).
  * (bsx_attn_plan takes one only where its partials need no more than those of the plan
  * over whole requests.) */
 int bsx_attn_plan_ws(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,

@@ -4,6 +4,7 @@ of every block is scheduled once, and split blocks' partial rows are packed with
 overlap.  Masks and shapes outside the rule keep a record per request, and the C entry
 point without a workspace size never needs more workspace than that plan."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -83,3 +84,33 @@ def test_rule_and_workspace_fallback():
     assert blk.float_ws_bytes == 0 or whole.block_batch == 0
     strict = _plan(qo, kv, 32, 8, ws=None)[0]
     assert strict.block_batch == 0 or strict.float_ws_bytes <= whole.float_ws_bytes
+
+
+def test_more_blocks_than_the_blob_holds():
+    """About 4000 blocks fill the blob of a small batch; from there on the plan keeps a
+    record per request, without the time that scheduling the blocks would take."""
+    assert _plan([64000], [64000], 64, 8)[0].block_batch == 4000
+    for qo in ([65536], [8192] * 8):
+        assert _plan(qo, qo, 64, 8)[0].block_batch == 0
+
+    def least(mode):
+        times = []
+        for _ in range(20):
+            t = time.perf_counter()
+            _plan([65536], [65536], 64, 8, mode=mode)
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    none = least(_lib.MASK_NONE)  # never takes blocks; the same plan otherwise
+    assert least(_lib.MASK_CAUSAL) < 2 * none + 1e-4
+
+
+def test_random_block_plans_fit_the_blob():
+    """The bound that admits blocks covers what the schedule then needs, near the limit too."""
+    rng = np.random.default_rng(8)
+    for _ in range(20):
+        n = int(rng.integers(1, 40))
+        qo = rng.integers(1, 2 * 64000 // n, size=n)
+        kv = qo + rng.integers(0, 5000, size=n)
+        p, blob, _, _ = _plan(qo, kv, 64, 8)
+        assert p.plan_ints <= len(blob)
