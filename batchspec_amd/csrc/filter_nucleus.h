@@ -30,6 +30,8 @@
 // A row whose bin does not list (ties), or whose threshold is not found in the bins or the
 // window, takes the exact search of filter_deferred_kernel (large_threshold), in one
 // workgroup.
+// Rows outside canon.h's domain (+inf, all -inf, scores past 2^31) give what one workgroup
+// per row gives; a row with a NaN has no defined result on either path.
 // P = 8 up to 128 rows, 4 up to 256, 2 up to 512: at most four workgroups per compute unit
 // (256 rows: 262 -> 76 us, 512 rows: 300 -> 125 us).
 #pragma once
@@ -133,7 +135,7 @@ __global__ void __launch_bounds__(kThreads) nucleus_stats_kernel(NucArgs a) {
   // Groups loaded at once: all of a lane's whole rounds for the usual vocabularies (the
   // pass is a few memory round trips long, not bandwidth).
   constexpr int U = DT == BSX_DTYPE_FP32 ? 4 : 8;
-  u32x4 held[U];  // 16-bit rows, one lane per thread: its first U groups, counted below
+  u32x4 held[U];  // bf16 rows, one lane per thread: its first U groups, counted below
 #pragma unroll
   for (int u = 0; u < LPT; ++u) {
     const int q = (int)threadIdx.x + kThreads * u;

@@ -74,6 +74,44 @@ def test_small_workspace_keeps_the_plan_over_requests():
     AP.check(out, ref[0])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_exact_workspace_cache_pair_and_strided_q(dtype):
+    """A block plan whose partials fill its workspace to the last byte, on separate K and V
+    caches, with queries that are a slice of a wider tensor and appended rows with a token
+    stride of their own, against the plain call in a large workspace."""
+    hq, hkv, d = 32, 8, 128
+    b = make_verify_batch(3, 0, 0, 0, hq, hkv, d, 16, dtype=dtype, scale=0.5, seed=51,
+                          qo_lens=np.array([128, 80, 5]), ctx=np.array([965, 2158, 1782]),
+                          device=DEV)
+    args = (b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, hq, hkv, d, 16)
+    big = bsx.BatchPrefillWithPagedKVCacheWrapper(
+        torch.empty(256 << 20, dtype=torch.uint8, device=DEV), "NHD")
+    big.plan(*args, causal=True, q_data_type=dtype)
+    p = big.plan_info
+    assert p.block_batch > 0 and p.num_split_requests > 0
+    cache = b.cache.clone()
+    out, lse = big.run(b.q, cache, return_lse=True, append_key=b.k_new, append_value=b.v_new)
+    need = big._blob_bytes + int(p.float_ws_bytes)
+    guard = 4096
+    ws = torch.full((need + guard,), 0x5A, dtype=torch.uint8, device=DEV)
+    exact = bsx.BatchPrefillWithPagedKVCacheWrapper(ws[:need], "NHD")
+    exact.plan(*args, causal=True, q_data_type=dtype)
+    assert exact.plan_info.block_batch == p.block_batch
+    n = b.q.shape[0]
+    wide = torch.zeros((n, hq + 2 * hkv, d), dtype=dtype, device=DEV)  # q, k and v of a layer
+    wide[:, :hq], wide[:, hq:hq + hkv], wide[:, hq + hkv:] = b.q, b.k_new, b.v_new
+    kv = (b.cache[:, 0].contiguous(), b.cache[:, 1].contiguous())
+    out1, lse1 = exact.run(wide[:, :hq], kv, return_lse=True, append_key=wide[:, hq:hq + hkv],
+                           append_value=wide[:, hq + hkv:])
+    torch.cuda.synchronize()
+    assert torch.equal(out1, out) and torch.equal(lse1, lse)
+    assert torch.equal(kv[0], cache[:, 0]) and torch.equal(kv[1], cache[:, 1])
+    assert bool((ws[need:] == 0x5A).all())
+    b.cache = cache
+    ref = AP.oracle_per_request(b, "causal")[None]
+    AP.check(out, ref[0], lse, ref[1])
+
+
 def _exact64(b, r):
     """float64 output [qo_len, heads, D] of request r (causal)."""
     q0, q1 = int(b.qo_indptr[r]), int(b.qo_indptr[r + 1])

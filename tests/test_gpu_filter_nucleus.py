@@ -5,7 +5,10 @@ changes (128, 256, 512), the shortest vocabulary of the path and the one below i
 which a canonical thread has 7, 8 and 9 whole rounds, a last partial group (fp32, V mod 8 =
 4), rows that are not 16-byte aligned, more than eight elements per draw lane; ties, rows
 whose threshold lies outside the bf16 key window (around zero, or in a row of two values),
-all-negative rows, -inf padding, and nearly certain rows."""
+all-negative rows, -inf padding, and nearly certain rows.  Rows and temperatures outside the
+statistics' domain (+inf, all -inf, scores past 2^31) give what the path with one workgroup
+per row gives (more than 512 rows); rows with a NaN, which have no distribution, give an id
+of the vocabulary or -1."""
 import numpy as np
 import pytest
 import torch
@@ -91,3 +94,47 @@ def test_chain_and_probs(dt, kind, B, k, V, onehot):
     p = S.get_sampling_probs(t.to(DEV), 0.9, 0, 0.7).cpu().numpy().reshape(-1, V)
     want = OAc.filtered_probs(t.float().numpy().reshape(-1, V), 0.7, 0, 0.9)
     np.testing.assert_array_equal(p, want.reshape(-1, V))
+
+
+SPECIAL = ["one +inf", "many +inf", "one nan", "all nan", "all -inf", "+inf and nan", "-inf but one",
+           "lowest", "plain"]
+
+
+def _special_rows(V, dtype):
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn((len(SPECIAL), V), generator=g) * 2
+    x[0, 7] = float("inf")
+    x[1, 3::1000] = float("inf")
+    x[2, V - 1] = float("nan")
+    x[3] = float("nan")
+    x[4] = float("-inf")
+    x[5, 100], x[5, 200] = float("nan"), float("inf")
+    x[6] = float("-inf")
+    x[6, V // 2] = 1.0
+    x = x.to(dtype)
+    x[7] = torch.finfo(dtype).min  # a mask of the type's lowest value
+    x[7, 5:9] = 1.0
+    return x
+
+
+@pytest.mark.parametrize("temperature", [0.8, 1e-9, 1e-30, 1e-38])
+@pytest.mark.parametrize("V", [20000, 20001])
+@pytest.mark.parametrize("dt", sorted(DT))
+def test_rows_outside_the_domain(dt, V, temperature):
+    print(f"nucleus special rows {dt} V={V} T={temperature}", flush=True)
+    x = _special_rows(V, DT[dt]).to(DEV)
+    n = len(SPECIAL)
+    rest = torch.zeros((513 - n, V), dtype=x.dtype, device=DEV)
+    rest[:, 0] = 9.0
+    more = torch.cat([x, rest])  # too many rows for the split path
+    u = torch.rand(513, generator=torch.Generator().manual_seed(5)).to(DEV)
+    nan = torch.tensor(["nan" in kind for kind in SPECIAL], device=DEV)
+    for top_p in (0.5, 0.95):
+        many = S.sample(more[:, None], top_p, 0, temperature, uniforms=u)[:n]
+        few = S.sample(x[:, None], top_p, 0, temperature, uniforms=u[:n].clone())
+        assert torch.equal(few[~nan], many[~nan]), (few.flatten().tolist(), many.flatten().tolist())
+        assert bool(((few >= -1) & (few < V)).all())
+        pm = S.get_sampling_probs(more[:, None], top_p, 0, temperature)[:n][~nan]
+        pf = S.get_sampling_probs(x[:, None], top_p, 0, temperature)[~nan]
+        assert torch.equal(pf.isnan(), pm.isnan())
+        assert torch.equal(pf.nan_to_num(nan=-1.0), pm.nan_to_num(nan=-1.0))
