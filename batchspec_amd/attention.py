@@ -515,8 +515,9 @@ class BatchPrefillWithPagedKVCacheWrapper:
         qo_indptr, batchspec/models/modules/kv_cache.py:47-84, as
         batchspec/models/modules/attention/standard.py:63-66 calls it) and attention sees
         them, as the update followed by run() does.  The plan's page table must already
-        count those tokens (insert_kv runs before the layers).  One launch: the
-        attention kernel writes the rows into the cache before reading them."""
+        count those tokens (insert_kv runs before the layers).  The attention kernel
+        writes the rows into the cache before reading them (plans over query blocks,
+        plan_info.block_batch > 0, in a launch of its own)."""
         plan = self._plan
         if plan is None:
             raise RuntimeError("plan() must be called before run()")

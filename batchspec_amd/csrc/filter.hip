@@ -2668,10 +2668,12 @@ static filt::SplitArgs split_args(const void* a, int64_t n_a, const void* b, int
   return sa;
 }
 
-// Top-p alone over at most kNucMaxRows rows (300 -> 125 us at 512 rows of 128256; above it
-// the workspace of the parts, about 36 KB per row, is not asked for and one workgroup per
-// row fills the device), and rows of at least kNucMinVocab logits, so that a lane has whole
-// rounds (shorter rows are a few rounds of one workgroup).
+// Top-p alone over at most kNucMaxRows rows, and rows of at least kNucMinVocab logits, so that
+// a lane has whole rounds (shorter rows are a few rounds of one workgroup).  The bound on rows
+// is one of workspace, of which the parts take about 36 KB per row of every filtered call (18
+// MB at 512 rows), not of time: sample() over rows of 128256 bf16 logits, one workgroup per row
+// / two: 512 rows 300 / 125 us, 513 279 / 158, 768 318 / 184, 1024 384 / 248 (fp32: 513 rows
+// 301 / 240, 1024 478 / 470).
 static bool nucleus_applies(int64_t rows, int64_t V, int top_k, float top_p) {
   return !(top_k > 0 && (int64_t)top_k < V) && top_p > 0.f && top_p < 1.f &&
          rows <= filt::kNucMaxRows && V >= filt::kNucMinVocab;

@@ -117,8 +117,10 @@ typedef struct {
                              long request, each with the kv tokens its rows can
                              see): qblocks_per_cta 4, num_qgroups 1.
                              0: one record per request                         */
-  int32_t part_rows;      /* block plans: rows per kv head of all partials (the
-                             partials are packed: slots count rows)            */
+  int32_t part_rows;      /* block plans: rows per kv head of all partials in the
+                             input dtype (the partials are packed: a slot is
+                             2 * its first row, + 1 where the partials are fp32
+                             and take two such rows per query row)             */
 } bsx_attn_plan_t;
 
 /* Size (int32 entries) of the host buffer bsx_attn_plan needs for its blob. */
@@ -221,8 +223,8 @@ int bsx_attn_plan_device(const bsx_attn_plan_t* plan, const int32_t* qo_indptr_d
  *   plan_blob_d the device copy of the plan blob
  *   float_ws_d at least plan->float_ws_bytes bytes (partial results of split
  *              requests); runs that share one workspace must not overlap in time.
- * Two kernel launches when the plan splits requests (attention, then the merge of
- * the partial results), one otherwise. */
+ * Two kernel launches when the plan splits requests or blocks (attention, then the
+ * merge of the partial results), one otherwise. */
 int bsx_attn_run(const bsx_attn_plan_t* plan, const int32_t* plan_blob_d,
                  void* float_ws_d, int dtype, const void* q_d, int64_t q_stride_tok,
                  const void* k_cache_d, const void* v_cache_d, int64_t page_stride,
@@ -235,9 +237,10 @@ int bsx_attn_run(const bsx_attn_plan_t* plan, const int32_t* plan_blob_d,
  * kv_cache) (standard.py:69).  Arguments of bsx_attn_run, plus the appended rows
  * k_new_d / v_new_d [total_qo, num_kv_heads, head_dim] (token strides in elements):
  * token i of request b goes to position kv_len_b - qo_len_b + i of the cache, where the
- * plan's page table already counts it.  One launch: each workgroup whose tiles reach a
- * request's appended rows first writes them (for its kv heads) into the cache, then reads
- * them back with the other rows.  Outputs and cache contents equal bsx_kv_append followed
+ * plan's page table already counts it.  Without a launch of its own: each workgroup whose
+ * tiles reach a request's appended rows first writes them (for its kv heads) into the cache,
+ * then reads them back with the other rows.  (Block plans, block_batch > 0, write the rows
+ * in a launch before the attention's: a block's tiles hold rows of other blocks.)  Outputs and cache contents equal bsx_kv_append followed
  * by bsx_attn_run; rows at negative positions (kv_len < qo_len) are skipped, as there. */
 int bsx_attn_run_append(const bsx_attn_plan_t* plan, const int32_t* plan_blob_d,
                         void* float_ws_d, int dtype, const void* q_d, int64_t q_stride_tok,

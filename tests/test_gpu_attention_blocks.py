@@ -130,15 +130,16 @@ def _exact64(b, r):
     return out
 
 
+@pytest.mark.parametrize("qo,ctx,split_there", [(512, 1024, 0), (300, 1000, 4)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_split_blocks_lose_no_precision(dtype):
-    """Query tokens whose block is split although the plan over requests runs their request
-    whole: the error against 64 bits is that of the unsplit output.  The parts add fp32
-    roundings (2^-24) to an output rounded to 2^-9 or 2^-12; the bound leaves 2% for the
+def test_split_blocks_lose_no_precision(dtype, qo, ctx, split_there):
+    """Query tokens of split blocks, where the plan over requests runs their request whole and
+    where it splits it too: the error against 64 bits is no larger than that plan's.  fp32 parts
+    add roundings of 2^-24 to an output rounded to 2^-9 or 2^-12; the bound leaves 2% for the
     softmax weights' rounding, which falls differently (a second rounding to the 16-bit
     type makes it about 1.2 times)."""
     b = make_verify_batch(4, 0, 0, 0, 32, 8, 128, 16, dtype=dtype, scale=0.5, seed=41,
-                          qo_lens=np.full(4, 512), ctx=np.full(4, 1024), device=DEV)
+                          qo_lens=np.full(4, qo), ctx=np.full(4, ctx), device=DEV)
     args = (b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, 32, 8, 128, 16)
 
     def planned(nbytes):
@@ -150,8 +151,9 @@ def test_split_blocks_lose_no_precision(dtype):
     blocks = planned(256 << 20)
     p = blocks.plan_info
     assert p.block_batch > 0 and p.num_split_requests > 0
-    whole = planned(blocks._blob_bytes)  # no room for partials
-    assert whole.plan_info.block_batch == 0 and whole.plan_info.num_split_requests == 0
+    whole = planned(blocks._blob_bytes + int(p.float_ws_bytes) - 1)  # no room for the partials
+    assert whole.plan_info.block_batch == 0
+    assert whole.plan_info.num_split_requests == split_there
     rec = blocks.plan_blob[p.off_merge_seqs:p.off_merge_seqs + 4 * p.num_split_requests]
     split = torch.zeros(b.q.shape[0], dtype=torch.bool, device=DEV)
     for _, _, q0, n in rec.reshape(-1, 4):

@@ -37,6 +37,11 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
     qo[0] = 700
     kv = np.maximum(0, rng.integers(-20, 3000, size=12) + qo)
     plan, blob, qoi, kvp = _plan(qo, kv, hq, hkv)
+    over, obl, _, _ = _plan(qo, kv, hq, hkv, ws=0)  # the plan over requests
+    split_there = np.zeros(len(qo), bool)
+    if over.block_batch == 0:
+        osegs = obl[over.off_segments:over.off_segments + 4 * over.num_segments].reshape(-1, 4)
+        split_there[osegs[osegs[:, 3] >= 0, 0]] = True
     g = hq // hkv
     n = plan.block_batch
     assert n > 0
@@ -65,10 +70,17 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
         if len(mine) == 1:
             assert mine[0, 3] == -1
         else:
+            r = int(np.searchsorted(qoi, seq[i, 0], side="right")) - 1
+            wide = not split_there[r]  # fp32: rounded once in the plan over requests
             for s in mine:
-                rows_used += list(range(s[3], s[3] + ql * g))
+                assert s[3] % 2 == wide
+                rows_used += list(range(s[3] // 2, s[3] // 2 + ql * g * (1 + wide)))
+    assert over.block_batch == 0
     assert sorted(rows_used) == list(range(plan.part_rows))
-    assert plan.float_ws_bytes == plan.part_rows * hkv * (128 * 4 + 4)  # fp32 partials
+    assert plan.float_ws_bytes == plan.part_rows * hkv * (128 * 2 + 4)
+    rec = blob[plan.off_merge_seqs:plan.off_merge_seqs + 4 * plan.num_split_requests]
+    for a, b, q0, n in rec.reshape(-1, 4):
+        assert a % 2 == b % 2 and (b - a) // 2 % (n * g * (1 + a % 2)) == 0
 
 
 def test_rule_and_workspace_fallback():
