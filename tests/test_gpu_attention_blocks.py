@@ -130,16 +130,16 @@ def _exact64(b, r):
     return out
 
 
-@pytest.mark.parametrize("qo,ctx,split_there", [(512, 1024, 0), (300, 1000, 4)])
+@pytest.mark.parametrize("n,qo,ctx,split_there", [(1, 2100, 0, 0), (4, 160, 3000, 4)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_split_blocks_lose_no_precision(dtype, qo, ctx, split_there):
+def test_split_blocks_lose_no_precision(dtype, n, qo, ctx, split_there):
     """Query tokens of split blocks, where the plan over requests runs their request whole and
     where it splits it too: the error against 64 bits is no larger than that plan's.  fp32 parts
     add roundings of 2^-24 to an output rounded to 2^-9 or 2^-12; the bound leaves 2% for the
     softmax weights' rounding, which falls differently (a second rounding to the 16-bit
     type makes it about 1.2 times)."""
-    b = make_verify_batch(4, 0, 0, 0, 32, 8, 128, 16, dtype=dtype, scale=0.5, seed=41,
-                          qo_lens=np.full(4, qo), ctx=np.full(4, ctx), device=DEV)
+    b = make_verify_batch(n, 0, 0, 0, 32, 8, 128, 16, dtype=dtype, scale=0.5, seed=41,
+                          qo_lens=np.full(n, qo), ctx=np.full(n, ctx), device=DEV)
     args = (b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, 32, 8, 128, 16)
 
     def planned(nbytes):
@@ -156,11 +156,30 @@ def test_split_blocks_lose_no_precision(dtype, qo, ctx, split_there):
     assert whole.plan_info.num_split_requests == split_there
     rec = blocks.plan_blob[p.off_merge_seqs:p.off_merge_seqs + 4 * p.num_split_requests]
     split = torch.zeros(b.q.shape[0], dtype=torch.bool, device=DEV)
-    for _, _, q0, n in rec.reshape(-1, 4):
-        split[int(q0):int(q0) + int(n)] = True
-    ref = torch.cat([_exact64(b, r) for r in range(4)])[split]
+    for _, _, q0, ql in rec.reshape(-1, 4):
+        split[int(q0):int(q0) + int(ql)] = True
+    ref = torch.cat([_exact64(b, r) for r in range(n)])[split]
     err = [float((w.run(b.q, b.cache).double()[split] - ref).norm() / ref.norm())
            for w in (whole, blocks)]
     print(f"split query tokens {int(split.sum())} of {len(split)}: relative error whole "
           f"{err[0]:.6f}, blocks {err[1]:.6f}", flush=True)
     assert err[1] <= 1.02 * err[0]
+
+
+def test_whole_blocks_equal_the_plan_over_requests():
+    """Chunks that neither plan splits: the same tiles in the same order, so the outputs of the
+    two plans are the same bits."""
+    b = make_verify_batch(4, 0, 0, 0, 32, 8, 128, 16, dtype=torch.bfloat16, scale=0.5, seed=42,
+                          qo_lens=np.full(4, 512), ctx=np.full(4, 1024), device=DEV)
+    args = (b.qo_indptr, b.kv_indptr, b.kv_indices, b.kv_last_page_len, 32, 8, 128, 16)
+    res = []
+    for graph in (False, True):  # graph mode keeps a record per request
+        kw = dict(use_cuda_graph=True, paged_kv_indices_buf=b.kv_indices.clone()) if graph else {}
+        w = bsx.BatchPrefillWithPagedKVCacheWrapper(
+            torch.empty(256 << 20, dtype=torch.uint8, device=DEV), "NHD", **kw)
+        w.plan(*args, causal=True, q_data_type=b.q.dtype)
+        assert (w.plan_info.block_batch == 0) == graph
+        n_seg = int(w.plan_blob[w.plan_info.off_seg_indptr + w.plan_info.num_ctas])
+        assert n_seg == (4 if graph else w.plan_info.block_batch)
+        res.append(w.run(b.q, b.cache, return_lse=True))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])

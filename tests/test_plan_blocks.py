@@ -37,11 +37,12 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
     qo[0] = 700
     kv = np.maximum(0, rng.integers(-20, 3000, size=12) + qo)
     plan, blob, qoi, kvp = _plan(qo, kv, hq, hkv)
-    over, obl, _, _ = _plan(qo, kv, hq, hkv, ws=0)  # the plan over requests
+    over, obl, _, _ = _plan(qo, kv, hq, hkv, ws=0)  # the plan over requests, if blocks split
     split_there = np.zeros(len(qo), bool)
     if over.block_batch == 0:
         osegs = obl[over.off_segments:over.off_segments + 4 * over.num_segments].reshape(-1, 4)
         split_there[osegs[osegs[:, 3] >= 0, 0]] = True
+    assert (over.block_batch > 0) == (plan.num_split_requests == 0)
     g = hq // hkv
     n = plan.block_batch
     assert n > 0
@@ -75,7 +76,6 @@ def test_blocks_cover_every_query_token_and_visible_tile(hq, hkv, seed):
             for s in mine:
                 assert s[3] % 2 == wide
                 rows_used += list(range(s[3] // 2, s[3] // 2 + ql * g * (1 + wide)))
-    assert over.block_batch == 0
     assert sorted(rows_used) == list(range(plan.part_rows))
     assert plan.float_ws_bytes == plan.part_rows * hkv * (128 * 2 + 4)
     rec = blob[plan.off_merge_seqs:plan.off_merge_seqs + 4 * plan.num_split_requests]
@@ -126,3 +126,37 @@ def test_random_block_plans_fit_the_blob():
         kv = qo + rng.integers(0, 5000, size=n)
         p, blob, _, _ = _plan(qo, kv, 64, 8)
         assert p.plan_ints <= len(blob)
+
+
+def _loads(plan, blob, cost):
+    seg = blob[plan.off_seg_indptr:plan.off_seg_indptr + plan.num_ctas + 1]
+    recs = blob[plan.off_segments:plan.off_segments + 4 * plan.num_segments].reshape(-1, 4)
+    return [sum(max(1, e - t) * cost[r] + 8 for r, t, e, _ in recs[a:b])
+            for a, b in zip(seg, seg[1:])]
+
+
+@pytest.mark.parametrize("qo,ctx,hq,hkv,whole", [
+    ([383, 300, 250, 383, 100], [0] * 5, 32, 8, True),   # short: whole blocks are even enough
+    ([512] * 4, [1024] * 4, 32, 8, True),
+    ([1352, 1100], [512, 0], 40, 8, True),               # several blocks a workgroup
+    ([450], [4096], 16, 8, False),                       # few long blocks
+    ([128] * 6 + [5] * 30, [3000] * 36, 28, 4, False),
+])
+def test_blocks_stay_whole_where_splitting_gains_little(qo, ctx, hq, hkv, whole):
+    qo = np.array(qo)
+    kv = qo + np.array(ctx)
+    plan, blob, _, _ = _plan(qo, kv, hq, hkv)
+    n = plan.block_batch
+    assert n > 0 and (plan.num_split_requests == 0) == whole
+    seq = blob[:4 * n].reshape(-1, 4)
+    waves = -(-seq[:, 1] * (hq // hkv) // 32)
+    cost = np.maximum(2, waves)
+    tiles = -(-seq[:, 2] // 32)
+    load = np.maximum(1, tiles) * cost + 8
+    share = -(-int(load.sum()) // (512 // hkv))
+    limit = lambda share: share + share // 4 + 64
+    if whole:
+        assert plan.float_ws_bytes == 0 and plan.num_segments == n
+        assert max(_loads(plan, blob, cost)) <= limit(max(share, 12))
+    else:
+        assert load.max() > limit(share)
